@@ -20,7 +20,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OUT = os.path.join(HERE, "libl3p.so")
 BUILD = os.path.join(HERE, "_build")
-SOURCES = ["gemv.hip", "gemm.hip", "blocks.hip", "layers.hip", "api.cpp", "model.cpp"]
+SOURCES = ["gemv.hip", "gemm.hip", "gemm_split.hip", "blocks.hip", "layers.hip", "api.cpp", "model.cpp"]
 ARCH = os.environ.get("L3P_ARCH", "gfx950")
 
 FLAGS = [f"--offload-arch={ARCH}", "-O3", "-std=c++17", "-fPIC", "-ffp-contract=off",
@@ -47,7 +47,7 @@ def _compile(src: str) -> str:
 
 def build() -> str:
     os.makedirs(BUILD, exist_ok=True)
-    with ThreadPoolExecutor(max_workers=min(4, len(SOURCES))) as ex:
+    with ThreadPoolExecutor(max_workers=min(8, len(SOURCES))) as ex:
         objs = list(ex.map(_compile, SOURCES))
     tmp = OUT + ".tmp"
     cmd = [hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", tmp, *objs]

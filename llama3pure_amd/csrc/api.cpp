@@ -228,14 +228,17 @@ int l3p_gemm_static(int type, const void* w, int rows, int cols, const float* x,
             return;
         }
         L3P_REQUIRE(gemm_mfma_supported(type), L3P_E_UNSUPPORTED, "gemm_static: type %d", type);
-        // the plan l3p_gemm takes with its context workspace, so the values
-        // are l3p_gemm's; its partials must fit the file-scope array
-        const GemmPlan plan = gemm_plan(j, kGemmWsFloats);
-        L3P_REQUIRE(plan.partial_floats <= kGemmStaticScratchFloats, L3P_E_UNSUPPORTED,
+        const GemmPlan tiles = gemm_plan(j, kGemmWsFloats);
+        L3P_REQUIRE(tiles.partial_floats <= kGemmStaticScratchFloats, L3P_E_UNSUPPORTED,
                     "gemm_static: %d x %d x batch %d needs %zu floats of split-K partials, more than the %zu of the "
                     "static scratch; use l3p_gemm",
-                    rows, cols, batch, plan.partial_floats, kGemmStaticScratchFloats);
-        launch_gemm_planned(j, plan, plan.nsplit > 1 || plan.streamk ? gemm_static_scratch() : nullptr, st);
+                    rows, cols, batch, tiles.partial_floats, kGemmStaticScratchFloats);
+        // the plan l3p_gemm takes with its context workspace, so the values
+        // are l3p_gemm's; its partials fit the file-scope array
+        const GemmPlan plan = gemm_split_supported(type) ? gemm_split_plan(j, kGemmWsFloats) : tiles;
+        float* ws = plan.partial_floats ? gemm_static_scratch() : nullptr;
+        if (gemm_split_supported(type)) launch_gemm_split(j, plan, ws, st);
+        else launch_gemm_planned(j, plan, ws, st);
     });
 }
 

@@ -195,10 +195,16 @@ struct GemmPlan {
     int nsplit = 1, ksteps = 0;   // stream-K: nsplit = most partial slots of a tile, ksteps = K steps of a tile
     int bn = 64;   // output columns per tile: 64, or 128 when those tiles fill the CUs unsplit
     int streamk = 0;   // > 0: stream-K over that many workgroups
+    int shape = 0;     // gemm_split.hip's tile shape
     size_t partial_floats = 0;
 };
 GemmPlan gemm_plan(const GemmJob& j, size_t ws_floats);
 void launch_gemm_planned(const GemmJob& j, const GemmPlan& plan, float* ws, hipStream_t s);
+// gemm_split.hip: the same product on the bf16 matrix cores (every type of
+// gemm_mfma_supported but F32), its plan and its launch
+bool gemm_split_supported(int type);
+GemmPlan gemm_split_plan(const GemmJob& j, size_t ws_floats);
+void launch_gemm_split(const GemmJob& j, const GemmPlan& plan, float* ws, hipStream_t s);
 // split-K partials of a context (allocated with it): 64 MB
 constexpr size_t kGemmWsFloats = (size_t)16 << 20;
 // the file-scope partials array of l3p_gemm_static (16 MB per GPU) and its
