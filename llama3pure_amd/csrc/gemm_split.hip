@@ -1,9 +1,45 @@
 // gemm_split.hip — the prefill GEMMs of the types the reference dequantizes
 // before its batched dot (matmul_deq_batch_4row, llama3pure-c-engine.c:
-// 2179-2273), on the bf16 matrix cores with fp32's precision:
+// 2179-2273; F32 weights: gemm.hip), on the bf16 matrix cores with fp32's
+// precision:
 //   Y[m][n] (=|+=) sum_k W[n][k] * X[m][k]
+//
+// Operands.  An integer code of at most 8 bits is a bf16 value, and the 24
+// significant bits of an fp32 x are three (truncations of 8 bits each, their
+// sum is x exactly), so three bf16 products give the exact code * x, summed in
+// fp32: Q8_0, Q4_K, Q5_K and Q6_K multiply their quants, Q3_K and Q2_K their
+// quants times the 6- or 4-bit group scale (at most 128), BF16 its values, F16
+// a high and a low part (six products).  The block's fp32 scale (d, or d times
+// the group's) multiplies the sum over its 32 (Q6_K: 16) columns.  Offsets
+// (Q4_K, Q5_K, Q2_K) are one more product per super-block: the groups' offset
+// codes times the groups' sums of x, split alike, times dmin.  Every weight
+// enters as exactly as before, and fewer fp32 additions follow it: against 64
+// bits the results lie closer than those of fp32 products summed column by
+// column.  x is scaled by 2^-14 and the results back, so that sums of codes
+// times x stay finite for every finite x (below 2^-98 in magnitude x's last
+// part is subnormal).
+//
+// Why.  The fp32 matrix cores do 256 FLOP a cycle and CU, the bf16 ones 4096:
+// three products are 3/16 of the time.  Q8_0 14336 x 4096 x 1024 rows: 966 ->
+// 388 us (125 -> 310 TFLOP/s).
+//
+// What bounds it.  MFMA and VALU issue add up (64 x 128 tiles: 38% and 59% of
+// the SIMDs' cycles, at a clock that falls from 2.4 to 1.7-2 GHz), so what
+// counts is VALU work per output: 7.5 operations an x and 1.5-4 a weight for
+// each tile that expands it, and one fused multiply-add per output and block.
+// A 128 x 256 tile, each of four waves 64 x 128, is the largest whose
+// accumulators leave room for two workgroups a CU.  Two LDS buffers with the
+// expansion between a wave's own MFMAs cost the second workgroup and were
+// slower (Q8_0 458 us, Q4_K 738).
+//
+// A workgroup walks K in steps of 32: x and weights of a step, fetched one step
+// earlier, go to LDS (80-byte rows), and each wave forms its 32 x 32 tiles with
+// v_mfma_f32_32x32x16_bf16, a tile's scaling issued beside the next tile's
+// products.  x fragments are held for one row of tiles and the weights' re-read:
+// holding all of x's spilled (Q6_K 703 -> 477 us).  Where the tiles are too few
+// for the CUs, K is cut in equal runs (multiples of a super-block where there
+// are offsets), whose fp32 partials gemm_reduce_kernel adds in order.
 #include <algorithm>
-#include <cstdlib>
 
 #include "device_common.h"
 #include "gemm_tiles.h"
@@ -29,7 +65,7 @@ struct WType {
     static constexpr int kUnit = kMinGroup ? 256 : kK;                 // K is cut at multiples of this
 };
 
-// |x| 2^-14: sums of 256 offset products (6-bit codes times sums of 32 x) stay finite for every finite x
+// sums of 256 columns' offset products (6-bit codes times sums of 32 x) stay finite for every finite x
 constexpr float kXScale = 1.0f / 16384, kXUnscale = 16384.0f;
 
 __device__ __forceinline__ uint32_t bits(float f) { return __float_as_uint(f); }
@@ -134,18 +170,16 @@ __device__ __forceinline__ void decode_codes(const WRaw& r, int e0, WSlice& o) {
     }
 }
 
-// x 2^-14 (or x) as three bf16 values whose sum it is: 24 significant bits in
-// three truncations of 8.
-template <bool kScale, bool kInf>
+// x 2^-14 as three bf16 values whose sum it is: 24 significant bits in three
+// truncations of 8.  The clamp lies above any finite remainder; an infinity
+// (or NaN), whose remainder is NaN, gets a finite second part, so its first
+// part decides.
 __device__ __forceinline__ void split_pair(float a, float b, uint32_t& p1, uint32_t& p2, uint32_t& p3) {
-    const float s = kScale ? kXScale : 1.0f;
-    const float xa = a * s, xb = b * s;
+    constexpr float kTop = 0x1p113f;
+    const float xa = a * kXScale, xb = b * kXScale;
     p1 = pack_high(xa, xb);
-    float ra = xa - high_half(xa), rb = xb - high_half(xb);
-    if constexpr (kInf) {   // an infinity is its first part alone
-        ra = fabsf(xa) == INFINITY ? 0.0f : ra;
-        rb = fabsf(xb) == INFINITY ? 0.0f : rb;
-    }
+    const float ra = __builtin_amdgcn_fmed3f(xa - high_half(xa), -kTop, kTop);
+    const float rb = __builtin_amdgcn_fmed3f(xb - high_half(xb), -kTop, kTop);
     p2 = pack_high(ra, rb);
     p3 = pack_high(ra - high_half(ra), rb - high_half(rb));
 }
@@ -206,20 +240,11 @@ __global__ void __launch_bounds__(256, OCC) gemm_split_kernel(GemmArgs a) {
         for (int u = 0; u < WU; ++u) fetch_slice<QT>(wr[u], wrow[u], k0 + 16 * (t & 1));
     };
     auto store = [&](int k0) {
-        float top = 0.0f;
-#pragma unroll
-        for (int u = 0; u < XU; ++u)
-            top = fmaxf(top, fmaxf(fmaxf(fabsf(xv[u].x), fabsf(xv[u].y)), fmaxf(fabsf(xv[u].z), fabsf(xv[u].w))));
-        const bool inf = __builtin_amdgcn_ballot_w64(top == INFINITY) != 0;
 #pragma unroll
         for (int u = 0; u < XU; ++u) {
             uint2 p[3];
-            split_pair<W::kScaled, false>(xv[u].x, xv[u].y, p[0].x, p[1].x, p[2].x);
-            split_pair<W::kScaled, false>(xv[u].z, xv[u].w, p[0].y, p[1].y, p[2].y);
-            if (inf) {
-                split_pair<W::kScaled, true>(xv[u].x, xv[u].y, p[0].x, p[1].x, p[2].x);
-                split_pair<W::kScaled, true>(xv[u].z, xv[u].w, p[0].y, p[1].y, p[2].y);
-            }
+            split_pair(xv[u].x, xv[u].y, p[0].x, p[1].x, p[2].x);
+            split_pair(xv[u].z, xv[u].w, p[0].y, p[1].y, p[2].y);
 #pragma unroll
             for (int c = 0; c < 3; ++c) *reinterpret_cast<uint2*>(&xs[c][(xr + 32 * u) * kLD + xc]) = p[c];
         }
@@ -232,7 +257,7 @@ __global__ void __launch_bounds__(256, OCC) gemm_split_kernel(GemmArgs a) {
                 if (W::kMinGroup == 32) s += dpp<0x141>(s);         // the other four of eight
                 if ((t & (W::kMinGroup / 4 - 1)) == 0) {
                     uint32_t p1, p2, p3;
-                    split_pair<true, true>(s, 0.0f, p1, p2, p3);
+                    split_pair(s, 0.0f, p1, p2, p3);
                     const int i = (xr + 32 * u) * NM + ((k0 + xc) & 255) / W::kMinGroup;
                     xm[0][i] = (uint16_t)p1;
                     xm[1][i] = (uint16_t)p2;
@@ -281,28 +306,23 @@ __global__ void __launch_bounds__(256, OCC) gemm_split_kernel(GemmArgs a) {
         if (k0 + kK < kend) fetch(k0 + kK);   // in flight during this step's matrix work
         // The wave's 32 x 32 tiles one after the other: a tile's products go to
         // b, and its scaling into acc runs in the shadow of the next tile's.
-        bf16x8 xf[TM][2][3];
-#pragma unroll
-        for (int im = 0; im < TM; ++im)
-#pragma unroll
-            for (int s = 0; s < 2; ++s)
-#pragma unroll
-                for (int c = 0; c < 3; ++c) xf[im][s][c] = frag(&xs[c][(mw + 32 * im + i32) * kLD + 16 * s + 8 * h]);
         floatx16 b[2];
         float sc[2];
 #pragma unroll
-        for (int in = 0; in < TN; ++in) {
-            const int n = nw + 32 * in + i32;
-            bf16x8 wf[2][W::kParts];
+        for (int im = 0; im < TM; ++im) {
+            bf16x8 xf[2][3];
 #pragma unroll
             for (int s = 0; s < 2; ++s)
 #pragma unroll
-                for (int c = 0; c < W::kParts; ++c) wf[s][c] = frag(&ws[c][n * kLD + 16 * s + 8 * h]);
-            float scale[NS];
+                for (int c = 0; c < 3; ++c) xf[s][c] = frag(&xs[c][(mw + 32 * im + i32) * kLD + 16 * s + 8 * h]);
 #pragma unroll
-            for (int s = 0; s < NS; ++s) scale[s] = dsc[s][n];
+            for (int in = 0; in < TN; ++in) {
+                const int n = nw + 32 * in + i32;
+                bf16x8 wf[2][W::kParts];
 #pragma unroll
-            for (int im = 0; im < TM; ++im) {
+                for (int s = 0; s < 2; ++s)
+#pragma unroll
+                    for (int c = 0; c < W::kParts; ++c) wf[s][c] = frag(&ws[c][n * kLD + 16 * s + 8 * h]);
                 if constexpr (!W::kScaled) {
 #pragma unroll
                     for (int s = 0; s < 2; ++s)
@@ -310,31 +330,30 @@ __global__ void __launch_bounds__(256, OCC) gemm_split_kernel(GemmArgs a) {
                         for (int c = 2; c >= 0; --c)
 #pragma unroll
                             for (int wc = W::kParts - 1; wc >= 0; --wc)
-                                acc[im][in] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xf[im][s][c], wf[s][wc],
+                                acc[im][in] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xf[s][c], wf[s][wc],
                                                                                      acc[im][in], 0, 0, 0);
                 } else {
 #pragma unroll
                     for (int g = 0; g < NS; ++g) {
                         constexpr int kChain = 2 / NS;               // slabs of 16 columns under one scale
-                        const int p = (in * TM + im) * NS + g;       // chain p; chain p - 1 is scaled beside it
+                        const int p = (im * TN + in) * NS + g;       // chain p; chain p - 1 is scaled beside it
                         b[p & 1] = floatx16{};
-                        sc[p & 1] = scale[g];
+                        sc[p & 1] = dsc[g][n];
 #pragma unroll
                         for (int s = g * kChain; s < (g + 1) * kChain; ++s)
 #pragma unroll
                             for (int c = 2; c >= 0; --c)
-                                b[p & 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xf[im][s][c], wf[s][0], b[p & 1], 0,
-                                                                                   0, 0);
+                                b[p & 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xf[s][c], wf[s][0], b[p & 1], 0, 0, 0);
                         if (p > 0) {
                             const int o = (p - 1) / NS;
 #pragma unroll
                             for (int r = 0; r < 16; ++r)
-                                acc[o % TM][o / TM][r] =
-                                    __builtin_fmaf(sc[(p - 1) & 1], b[(p - 1) & 1][r], acc[o % TM][o / TM][r]);
+                                acc[o / TN][o % TN][r] =
+                                    __builtin_fmaf(sc[(p - 1) & 1], b[(p - 1) & 1][r], acc[o / TN][o % TN][r]);
                         }
 #pragma unroll
                         for (int i = 0; i < 3 * kChain; ++i) {
-                            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);               // one MFMA,
+                            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                       // one MFMA,
                             __builtin_amdgcn_sched_group_barrier(0x002, 16 / (3 * kChain) + 1, 0);   // then VALU
                         }
                     }
@@ -388,7 +407,7 @@ __global__ void __launch_bounds__(256, OCC) gemm_split_kernel(GemmArgs a) {
             for (int r = 0; r < 16; ++r) {
                 const int m = m0 + mw + 32 * im + 8 * (r >> 2) + 4 * h + (r & 3);
                 if (m >= a.m) continue;
-                const float v = acc[im][in][r];
+                const float v = W::kScaled ? acc[im][in][r] : acc[im][in][r] * kXUnscale;
                 if (P) {
                     P[(size_t)m * a.ntot + n] = v;
                 } else {
@@ -399,19 +418,19 @@ __global__ void __launch_bounds__(256, OCC) gemm_split_kernel(GemmArgs a) {
         }
 }
 
-// The tile shapes: 64 x 128 and 64 x 256 for most jobs; 128 x 256, which
-// fetches least per output, while its 256 registers a lane hold a type's slices
-// (not the K-quants': 0.60-0.64 us a step and 64 x 128 tile there, 0.75-1.0
-// spilled); 32 x 128 for few rows, or few tiles and long K.
+// The tile shapes.  128 x 256 expands fewest values per output and wins full
+// grids (14336 x 4096 x 1024: Q8_0 388 us against 449 and 461 of 64 x 128 and
+// 64 x 256, Q6_K 477 / 570 / 619), but with super-block offsets its 256
+// registers a lane do not hold the slices (Q4_K 922 / 550 / 543), so those types
+// have the first three; 32 x 128 is for few rows (1000 x 2304 x 37: 15.0 against
+// 16.5) and 64 x 128 for what leaves CUs idle otherwise.
 struct Shape {
     int bm, bn;
     float alone, step;   // us of a K step of one workgroup: a CU to itself; its share of a full CU (Q8_0, measured)
 };
-constexpr Shape kShapes[4] = {{32, 128, 0.65f, 0.35f}, {64, 128, 0.83f, 0.47f}, {64, 256, 1.24f, 0.90f},
-                              {128, 256, 2.4f, 1.5f}};
-template <int QT>
-constexpr bool has_large() { return QT == L3P_Q8_0 || QT == L3P_BF16 || QT == L3P_F16; }
-int shapes_of(int type) { return type == L3P_Q8_0 || type == L3P_BF16 || type == L3P_F16 ? 4 : 3; }
+constexpr Shape kShapes[4] = {{32, 128, 0.66f, 0.35f}, {64, 128, 0.82f, 0.47f}, {64, 256, 1.25f, 0.92f},
+                              {128, 256, 1.85f, 1.45f}};
+constexpr bool has_offsets(int type) { return type == L3P_Q2_K || type == L3P_Q4_K || type == L3P_Q5_K; }
 
 template <int QT>
 void launch_type(const GemmArgs& a, int shape, int grid, hipStream_t st) {
@@ -420,12 +439,12 @@ void launch_type(const GemmArgs& a, int shape, int grid, hipStream_t st) {
     case 1: launch_kernel(gemm_split_kernel<QT, 64, 128, 2, 3>, dim3(grid), dim3(256), 0u, st, a); break;
     case 2: launch_kernel(gemm_split_kernel<QT, 64, 256, 2, 2>, dim3(grid), dim3(256), 0u, st, a); break;
     default:
-        if constexpr (has_large<QT>())
+        if constexpr (!has_offsets(QT))
             launch_kernel(gemm_split_kernel<QT, 128, 256, 2, 2>, dim3(grid), dim3(256), 0u, st, a);
     }
 }
 
-int unit_of(int type) { return type == L3P_Q2_K || type == L3P_Q4_K || type == L3P_Q5_K ? 256 : kK; }
+int unit_of(int type) { return has_offsets(type) ? 256 : kK; }
 
 }  // namespace
 
@@ -441,23 +460,19 @@ GemmPlan gemm_split_plan(const GemmJob& j, size_t ws_floats) {
     // l3p_gemm's values: for them the partials of this plan fit it too
     if (ws_floats > kGemmStaticScratchFloats && gemm_plan(j, ws_floats).partial_floats <= kGemmStaticScratchFloats)
         ws_floats = kGemmStaticScratchFloats;
-    const int force = getenv("L3P_SPLIT_SHAPE") ? atoi(getenv("L3P_SPLIT_SHAPE")) : -1;
-    const int forcez = getenv("L3P_SPLIT_Z") ? atoi(getenv("L3P_SPLIT_Z")) : -1;
-    for (int s = 0; s < shapes_of(j.type); ++s) {
+    for (int s = 0; s < (has_offsets(j.type) ? 3 : 4); ++s) {
         const Shape& sh = kShapes[s];
-        if (force >= 0 && force != s) continue;
         long tiles = 0;
         for (int i = 0; i < j.nseg; ++i) tiles += (j.seg[i].n + sh.bn - 1) / sh.bn;
         tiles *= (j.m + sh.bm - 1) / sh.bm;
         for (int z = 1; z <= 32 && z <= units; ++z) {
             const int run = (units + z - 1) / z, runs = (units + run - 1) / run;   // no empty run
             if (runs != z) continue;
-            if (forcez > 0 && z != forcez) continue;
             const size_t partial = z > 1 ? (size_t)z * j.m * ntot : 0;
             if (partial > ws_floats) break;
             const float n = (float)((tiles * z + cus - 1) / cus);   // workgroups a CU runs
             float us = std::max(sh.alone, n * sh.step) * (float)(run * (unit / kK));
-            if (z > 1) us += 3.0f + 0.15f * z + (float)partial * 8.0f / 4e6f;   // write, read and one more launch
+            if (z > 1) us += 3.0f + 0.1f * z + (float)partial * 8.0f / 6e6f;   // write, read and one more launch
             if (us < best_us) {
                 best_us = us;
                 best.shape = s;
@@ -505,6 +520,9 @@ void launch_gemm_split(const GemmJob& j, const GemmPlan& plan, float* ws, hipStr
     a.nsplit = plan.nsplit;
     a.bn = sh.bn;
     a.part = a.nsplit > 1 ? ws : nullptr;
+    // every K run must hold at least one step: the kernel's loads start before its loop
+    L3P_REQUIRE(plan.ksteps > 0 && (long)(plan.nsplit - 1) * plan.ksteps * kK < j.k, L3P_E_INVALID,
+                "gemm: plan of %d runs of %d steps for %d columns", plan.nsplit, plan.ksteps, j.k);
     const long grid = (long)tiles * ((j.m + sh.bm - 1) / sh.bm) * plan.nsplit;
     L3P_REQUIRE(grid < (1L << 31), L3P_E_INVALID, "gemm: %ld workgroups", grid);
     switch (j.type) {
