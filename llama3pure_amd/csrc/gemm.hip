@@ -6,7 +6,9 @@
 // (matmul_deq_batch_4row, c:2179-2273) the fp32 matrix cores multiply every
 // weight expanded exactly to fp32 (dequantize_row_*, c:611-934) with the fp32
 // activation, so the products are the reference's and only the fp32
-// summation order differs.  For the types whose batched dot takes Q8_0
+// summation order differs (only F32 weights still come here: gemm_split.hip
+// takes the others, and l3p_gemm_static's limits follow this plan for all).
+// For the types whose batched dot takes Q8_0
 // activations (Q4_0, Q4_1, Q5_0, Q5_1, IQ4_NL) the int8 matrix cores form
 // the exact block dots (the int8 section further down).
 //

@@ -751,7 +751,7 @@ struct RowsOut {
 
 // y rows (=|+=) W . x rows for `rows` prompt tokens, for one to three
 // matrices over the same x rows.  Matrices of one type and width run as one
-// GEMM launch (label `what`): the fp32 matrix-core GEMM for the types the
+// GEMM launch (label `what`): the split bf16 (F32: fp32) GEMM for the types the
 // reference dequantizes, the int8 one for the Q8_0-activation types (the
 // reference's exact integer block dots, matmul_quantized_batch, c:2305-2318).
 static bool gemm_capable(int type) { return gemm_mfma_supported(type) || gemm_q8_activation(type); }
