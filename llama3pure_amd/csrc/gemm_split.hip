@@ -444,10 +444,6 @@ void launch_type(const GemmArgs& a, int shape, int grid, hipStream_t st) {
     }
 }
 
-// Types with offsets keep a K to here whole.  Cut, it is faster (Q5_K 512 x 512 x
-// 11: 12.1 us, whole 16.5, on fp32 20.2), but its rounding then turns a near-tie
-// of the small Q5_K model's greedy decode the other way than the reference.
-constexpr int kUncut = 1024;
 int unit_of(int type) { return has_offsets(type) ? 256 : kK; }
 
 }  // namespace
@@ -474,7 +470,11 @@ GemmPlan gemm_split_plan(const GemmJob& j, size_t ws_floats) {
             if (runs != z) continue;
             const size_t partial = z > 1 ? (size_t)z * j.m * ntot : 0;
             if (partial > ws_floats) break;
-            if (z > 1 && has_offsets(j.type) && j.k <= kUncut) break;
+            // Runs of types with offsets have two super-blocks or more: one is
+            // faster still (Q5_K 512 x 512 x 11: 12.1 us, two 16.5, fp32 20.5), but
+            // its rounding turns a near-tie of the small Q5_K model's greedy decode
+            // the other way than the reference.
+            if (z > 1 && has_offsets(j.type) && run < 2) break;
             const float n = (float)((tiles * z + cus - 1) / cus);   // workgroups a CU runs
             float us = std::max(sh.alone, n * sh.step) * (float)(run * (unit / kK));
             if (z > 1) us += 3.0f + 0.1f * z + (float)partial * 8.0f / 6e6f;   // write, read and one more launch

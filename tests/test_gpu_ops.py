@@ -424,6 +424,59 @@ def test_gemm_stream_k_overrides(ctx, torch_gpu, cpuref, env, monkeypatch):
     assert np.all(err <= tol), f"max err/tol {np.max(err / np.maximum(tol, 1e-30)):.3g}"
 
 
+@pytest.mark.parametrize("qtype", [t for t in GEMM_TYPES if t != l3p.F32])
+@pytest.mark.parametrize("rows,batch", [(1, 1), (127, 32), (129, 33), (257, 129), (4100, 1000)])
+def test_gemm_split_edges(ctx, torch_gpu, cpuref, qtype, rows, batch):
+    """The split bf16 products at the edges of their tiles (32, 64 and 128
+    batch rows by 128 and 256 weight rows), one and two super-blocks of K (or
+    one K step, and three, for the types without), against float64 within the
+    fp32 summation bound; x spans 2^-60..2^60 down its columns' magnitudes, so
+    every part of the three-way split counts."""
+    for cols in ((256, 512) if qtype in K_QUANTS else (32, 96)):
+        w = synth.random_blocks(qtype, rows, cols, seed=rows + cols)
+        xb = synth.random_x(cols, seed=batch, batch=batch).reshape(batch, cols)
+        xb = (xb * np.exp2(np.linspace(-60, 60, batch))[:, None]).astype(np.float32)
+        y = torch_gpu.full((batch * rows,), float("nan"), dtype=torch_gpu.float32, device="cuda")
+        ctx.gemm(qtype, dev(torch_gpu, w), rows, cols, dev(torch_gpu, xb), batch, cols, y, rows)
+        ctx.synchronize()
+        got = y.cpu().numpy().reshape(batch, rows)
+        W, A = _dequant_bound(cpuref, qtype, w, rows, cols)
+        x64 = xb.astype(np.float64)
+        err = np.abs(got - x64 @ W.T)
+        tol = gamma(cols + 4) * (np.abs(x64) @ A.T)
+        assert np.all(err <= tol), f"{cols} columns: max err/tol {np.max(err / np.maximum(tol, 1e-300)):.3g}"
+
+
+@pytest.mark.parametrize("qtype", [l3p.Q8_0, l3p.Q4_K, l3p.BF16])
+def test_gemm_split_large_and_infinite_x(ctx, torch_gpu, cpuref, qtype):
+    """x at the ends of fp32's range: the largest finite value gives the
+    product with the weight (or fp32's overflow of it), an infinity gives an
+    infinity of the weight's sign (NaN where the weight is 0) and NaN gives
+    NaN, in the rows that hold them and in no other."""
+    rows, cols = 130, 256
+    w = synth.random_blocks(qtype, rows, cols, seed=3)
+    W = np.stack([cpuref.dequant(qtype, w[r], cols) for r in range(rows)]).astype(np.float64)
+    x = np.zeros((4, cols), np.float32)
+    big = np.finfo(np.float32).max
+    x[0, 5], x[1, 37], x[2, 200], x[3, 7] = big, np.inf, np.nan, 1.0
+    y = empty_f32(torch_gpu, 4 * rows)
+    ctx.gemm(qtype, dev(torch_gpu, w), rows, cols, dev(torch_gpu, x), 4, cols, y, rows)
+    ctx.synchronize()
+    got = y.cpu().numpy().reshape(4, rows)
+    want = W[:, 5] * float(big)
+    fits = np.abs(want) < 0.999 * float(big)
+    assert fits.any()
+    # one product, rounded once (Q4_K: the group's product and its offset's): 2 ulp of the larger term
+    scale = np.abs(want) + (np.abs(W).max() * float(big) if qtype == l3p.Q4_K else 0)
+    assert np.all(np.abs(got[0][fits].astype(np.float64) - want[fits]) <= 2.0 ** -21 * scale[fits])
+    if qtype != l3p.Q4_K:   # (its code and offset terms are infinities of opposite signs: NaN either way it is written)
+        sure = W[:, 37] != 0
+        assert np.array_equal(got[1][sure], np.where(W[sure, 37] > 0, np.inf, -np.inf).astype(np.float32))
+    assert not np.isfinite(got[1][W[:, 37] != 0]).any()
+    assert np.isnan(got[2]).all()
+    assert np.array_equal(got[3], W[:, 7].astype(np.float32))
+
+
 def test_gemm_mfma_equals_gemv_within_bound(ctx, torch_gpu, cpuref):
     """The batched and the single-row forms agree within the same bound."""
     qtype, rows, cols, batch = l3p.Q8_0, 4096, 4096, 5
